@@ -217,6 +217,8 @@ __device__ __forceinline__ double ref_d2(const Box& b, d3 lo, d3 hi) {
 // within tol of a cutoff, some one in 10^5, is evaluated the reference's way
 // (nim_search), so the pair set is the reference's to the bit.  The near / far
 // classification needs no such care: either kernel may take a pair.
+// A distance that is not a number is a pair, as in the reference, and a near one: the
+// FP64 path lists every partner as near and reads its slots from the start only.
 // Bound by instructions: about 60 vector ones per 64 candidates.  32,768 waters at
 // 1.4 nm: 109 us (156 with FP64 distances and every group's cursors in vector
 // registers); 128 x 4,000 waters at 1.2 nm: 1,041 us (1,544).
@@ -429,7 +431,7 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
                         const double d2 = r.x * r.x + r.y * r.y + r.z * r.z;
                         in = !(d2 > c2l);
                         lng = d2 > c2s;
-                        near = d2 < near_r2;
+                        near = !(d2 >= near_r2);
                     }
                     in = in && valid && cm != ck_t;
                     const bool sol_m = cm - cg_off < nsol;

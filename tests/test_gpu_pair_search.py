@@ -63,3 +63,23 @@ def test_exact_lattice_ties():
     # spacing L / 4: partners at exactly half the box along the axes, within the cutoff
     s = gen.spc_water_box(64, box=1.6, seed=1, jitter=0.0, rcutp=0.8, rcutl=0.9, temperature=0.0)
     assert sets(s) > 100
+
+
+@pytest.mark.parametrize("prec", [rt.FP64, rt.MIXED])
+@pytest.mark.parametrize("boundary", ["vacuum", "triclinic"])
+def test_non_finite_point_in_a_one_cell_box(prec, boundary):
+    """one molecule lost, in lists with room to spare: every other one has it as a partner, nothing else changes"""
+    s = gen.water_truncoct(3) if boundary == "triclinic" else gen.spc_water_box(27, box=2.6, seed=2, temperature=0.0)
+    if boundary == "vacuum":
+        s.boundary = 0
+    ds = rt.DeviceSystem(s, precision=prec, use_settle=False)
+    ds.forcefield_apply()
+    n = len(ds.pairlist()["solvent_short"])
+    x = s.pos.copy()
+    x[:3, 1] = np.nan
+    for _ in range(2):
+        ds.set_state(x)
+        f = ds.forcefield_apply()["forces"]
+        assert not np.any(np.abs(f).max(axis=-1).reshape(-1, 3).max(axis=-1) < 1e6)
+        assert len(ds.pairlist()["solvent_short"]) >= n
+    ds.close()
