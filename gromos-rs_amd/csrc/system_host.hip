@@ -1626,8 +1626,11 @@ SysPtrs gromos_amd_system::ptrs() const {
     p.sol_order = d_sol_order;
     p.nsol_small = nsol_small;
     p.has_pert = has_pert ? 1 : 0;
-    p.any_rect = p.any_other = 0;
-    for (const JobDev& J : jobs) (J.box.kind == 1 ? p.any_rect : p.any_other) = 1;
+    p.any_rect = p.any_other = p.pert_twin = 0;
+    for (const JobDev& J : jobs) {
+        (J.box.kind == 1 ? p.any_rect : p.any_other) = 1;
+        if (J.has_pert && J.twin) p.pert_twin = 1;
+    }
     p.s2o = d_s2o;
     p.s_atom_cg = d_s_atom_cg;
     p.s_type = d_s_type;

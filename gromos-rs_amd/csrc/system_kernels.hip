@@ -2114,9 +2114,9 @@ __device__ __forceinline__ void gen_atom32(const SysPtrs& p, int32_t a, int32_t 
     int32_t ta = p.s_type[a];
     bool cgp = J.use_cg_grouped != 0 && !LONG;
     const bool jp = PERT && !LONG && J.has_pert;
-    // SOLV (a solvent atom's lane): solvent atoms are never perturbed, so the
-    // lane never evaluates a perturbed pair (its first atom's lanes do both
-    // shares) and carries no FP64 soft-core code
+    // SOLV (a solvent atom's lane): solvent atoms are never perturbed; of a listed
+    // pair with a perturbed first atom the lane takes its own share in FP32, and
+    // of a cached long one its correction in FP64 outside this function (k_gen_sv)
     const bool po = !SOLV && jp && p.pflag[o];
     PertAtom PA{};
     if (po) PA = pert_atom(p, J, o);
@@ -2276,8 +2276,11 @@ __device__ __forceinline__ void gen_atom32(const SysPtrs& p, int32_t a, int32_t 
 // those pairs' energies and virial belong to the solute atom's block
 // (k_gen_sol): these lanes add none.  (Run beside the solvent pair kernel into
 // a per-group buffer added afterwards, it measured slower: 2.25e11 against
-// 2.33e11 pairs/s on the 64-job FEP mix.)
-template <int GSV_LANES, bool PERT>
+// 2.33e11 pairs/s on the 64-job FEP mix.)  TWIN: the batch has twin-range jobs with
+// perturbed atoms, whose cached long pairs are corrected every step at the current
+// positions, the solvent atoms' share here (FP64, an instantiation of its own for
+// its registers).
+template <int GSV_LANES, bool PERT, bool TWIN>
 __global__ void __launch_bounds__(BLOCK) k_gen_sv(SysPtrs p, int32_t ngsol) {
     constexpr int GSV_SLOT = 4 * GSV_LANES;   // solvent molecules have at most 4 atoms
     const int32_t w = ((int32_t)blockIdx.x * BLOCK + (int32_t)threadIdx.x) / GSV_SLOT;
@@ -2291,6 +2294,21 @@ __global__ void __launch_bounds__(BLOCK) k_gen_sv(SysPtrs p, int32_t ngsol) {
         if (i < p.s_cg_n[k] && !held(p, p.atom_job[p.s2o[sk]])) a = sk + i;
     }
     if (a >= 0) gen_atom32<false, false, true, PERT>(p, a, p.s2o[a], c, GSV_LANES, v, fx, fy, fz);
+    if (TWIN && a >= 0) {
+        const int32_t o = p.s2o[a];
+        const JobDev& J = p.jobs[p.atom_job[o]];
+        int32_t e0 = 0, e1 = 0;
+        if (J.has_pert && J.twin) gen_range(p, p.s_atom_cg[a], true, e0, e1);
+        for (int32_t e = e0 + c; e < e1; e += GSV_LANES) {
+            const uint32_t ent = p.gen_ent[e];
+            if (!(ent & ENT_LONG) || (ent & (ENT_CANON | ENT_VVLONG))) continue;
+            const int32_t m = (int32_t)(ent & ENT_IDX), sm = p.s_cg_start[m], nm = p.s_cg_n[m];
+            for (int32_t b = 0; b < nm; ++b) {
+                const int32_t ob = p.s2o[sm + b];
+                if (p.pflag[ob]) pert_pair_delta(p, J, ob, o, false, v, fx, fy, fz);
+            }
+        }
+    }
 #pragma unroll
     for (int m = 1; m < GSV_LANES; m <<= 1) {
         fx += __shfl_xor(fx, m, WAVE);
@@ -3822,8 +3840,9 @@ void launch_gen(const SysPtrs& p, int32_t npad, bool lng, int32_t virial, int32_
         constexpr int32_t GPB = BLOCK / (4 * 2);   // groups per block
         const dim3 g((unsigned)((ngsol + GPB - 1) / GPB));
         if (solv && ngsol > 0) {
-            if (pert) hipLaunchKernelGGL((k_gen_sv<2, true>), g, dim3(BLOCK), 0, s, p, ngsol);
-            else hipLaunchKernelGGL((k_gen_sv<2, false>), g, dim3(BLOCK), 0, s, p, ngsol);
+            if (p.pert_twin) hipLaunchKernelGGL((k_gen_sv<2, true, true>), g, dim3(BLOCK), 0, s, p, ngsol);
+            else if (pert) hipLaunchKernelGGL((k_gen_sv<2, true, false>), g, dim3(BLOCK), 0, s, p, ngsol);
+            else hipLaunchKernelGGL((k_gen_sv<2, false, false>), g, dim3(BLOCK), 0, s, p, ngsol);
         }
         if (solu) {
             if (virial && pert) GAMD_SOL(false, true, true, true, 1);

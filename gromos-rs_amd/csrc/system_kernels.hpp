@@ -46,6 +46,7 @@ struct SysPtrs {
     const int32_t* sol_order;      // solute indices: the small solutes' atoms, then the large ones'
     int32_t nsol_small;            // of the first kind (SOL_WAVE_MIN)
     int32_t has_pert;              // the batch has perturbed atoms
+    int32_t pert_twin;             // ... in a job with a twin range
     int32_t any_rect, any_other;   // the batch holds jobs with a rectangular / another boundary
     int4* s_fix;               // per sorted group: reference point as box fractions (k_nbl), original group
     int32_t* s2o;
