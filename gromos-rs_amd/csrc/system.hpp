@@ -39,6 +39,7 @@ struct JobDev {
     double c2s, c2l;                       // (rc + skin)^2 short / long
     double sv_c6[16], sv_c12[16], sv_qq[16];  // solvent template tables (innerloops.rs:241-255)
     double sv_q[4];                        // solvent template charges
+    int32_t neutral;                       // ... sum to zero exactly (the solvent pair kernels' form)
     Lambda lp;
     int32_t n_types, lj_off;
     int32_t use_cg_grouped;                // forcefield.rs:271-283

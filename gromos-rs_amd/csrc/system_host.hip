@@ -708,18 +708,24 @@ int layout_batch(gromos_amd_system* S, const std::vector<const JobImage*>& imgs,
             for (int i = 0; i < J.aps; ++i)
                 for (int jj = 0; jj < J.aps; ++jj)
                     if ((i || jj) && (J.sv_c6[i * 4 + jj] != 0.0 || J.sv_c12[i * 4 + jj] != 0.0)) S->vv_lj00 = 0;
-    // neutral solvent molecules (the charges of one molecule sum to zero exactly)
-    S->vv_neutral = 1;
-    for (const JobImage* im : imgs)
-        if (im->solvent) {
-            const int32_t f = im->J.n_solute_atoms, a = im->J.aps;
+    // the jobs' kinds of solvent molecules: neutral (the charges of one molecule sum
+    // to zero exactly) or not; GROMOS_AMD_VV_PAIRWISE_RF=1 takes every one as
+    // charged, whose RF form is per atom pair (checks)
+    const char* rf_env = std::getenv("GROMOS_AMD_VV_PAIRWISE_RF");
+    const bool pairwise = rf_env && std::atoi(rf_env) == 1;
+    S->vv_kinds = 0;
+    for (int j = 0; j < njobs; ++j)
+        if (imgs[j]->solvent) {
+            JobDev& J = S->jobs[j];
             double sum = 0.0;
-            for (int i = 0; i < a; ++i) sum += im->q[f + i];
-            if (sum != 0.0) S->vv_neutral = 0;
+            for (int i = 0; i < J.aps; ++i) sum += J.sv_q[i];
+            J.neutral = !pairwise && sum == 0.0;
+            S->vv_kinds |= J.neutral ? VV_NEUTRAL : VV_CHARGED;
         }
-    // GROMOS_AMD_VV_PAIRWISE_RF=1: the per-atom-pair RF form everywhere (checks)
-    if (const char* env = std::getenv("GROMOS_AMD_VV_PAIRWISE_RF"))
-        if (std::atoi(env) == 1) S->vv_neutral = 0;
+    // jobs without solvent (their groups' records are zeros) go with a kind there is
+    if (!S->vv_kinds) S->vv_kinds = VV_NEUTRAL;
+    for (int j = 0; j < njobs; ++j)
+        if (!imgs[j]->solvent) S->jobs[j].neutral = (S->vv_kinds & VV_NEUTRAL) ? 1 : 0;
     S->cell_bits = 1;
     while ((1ll << S->cell_bits) < (int64_t)S->ncell + 1) S->cell_bits++;
     S->n_papairs = (int32_t)papairs.size() / 4;
@@ -1152,8 +1158,8 @@ static std::map<int64_t, int32_t> g_tuned;
 static int tune_vv(gromos_amd_system* S, const SysPtrs& p, int32_t aps, int32_t mixed) {
     int32_t bucket = 0;
     while ((1 << bucket) < S->ncg) ++bucket;
-    const int32_t form = (S->vv_lj00 ? VV_LJ00 : 0) | (S->vv_neutral ? VV_NEUTRAL : 0);
-    int64_t key = (((((int64_t)bucket * 8 + aps) * 2 + mixed) * 4 + form) * 2 + S->do_virial);
+    const int32_t form = (S->vv_lj00 ? VV_LJ00 : 0) | S->vv_kinds;
+    int64_t key = (((((int64_t)bucket * 8 + aps) * 2 + mixed) * 8 + form) * 2 + S->do_virial);
     if (S->vv_lanes && S->tuned_key == key) return 0;
     if (const char* env = std::getenv("GROMOS_AMD_VV_LANES")) {
         int v = std::atoi(env);
@@ -1269,7 +1275,7 @@ int forcefield(gromos_amd_system* S, bool assemble) {
     hipEvent_t e0 = tl.a0, e1 = tl.a1, n0 = tl.n0, n1 = tl.n1;
     const int32_t aps = solvent_aps(S);
     if (int rc = tune_vv(S, p, aps, mixed)) return rc;
-    const int32_t form = (S->vv_lj00 ? VV_LJ00 : 0) | (S->vv_neutral ? VV_NEUTRAL : 0);
+    const int32_t form = (S->vv_lj00 ? VV_LJ00 : 0) | S->vv_kinds;
     // mixed md step: the near solvent pairs (FP64) and the solute atoms' pass
     // (general pairs, then excluded / 1-4 terms, covalent terms) are independent
     // of the far solvent pair kernel (separate outputs, inputs ready at the fork),
@@ -1340,7 +1346,7 @@ static int launch_step_graph(gromos_amd_system* S) {
     const SysPtrs p = S->ptrs();
     const int32_t mixed = S->precision == GROMOS_AMD_MIXED;
     const int32_t aps = solvent_aps(S);
-    const int32_t form = (S->vv_lj00 ? VV_LJ00 : 0) | (S->vv_neutral ? VV_NEUTRAL : 0);
+    const int32_t form = (S->vv_lj00 ? VV_LJ00 : 0) | S->vv_kinds;
     const int64_t shape[11] = {S->ncg, S->npad, S->njobs, S->nsol, S->vv_lanes, form, S->do_virial, S->twin ? 1 : 0,
                                mixed, aps, (int64_t)S->host_counters[4]};
     auto& g = S->graphs[S->cur];

@@ -720,6 +720,14 @@ __device__ __forceinline__ void shift32(const Box& b, d3 A, d3 B, float& x, floa
 // batch change; the integrator keeps its state): its pair kernels skip it.
 __device__ __forceinline__ bool held(const SysPtrs& p, int32_t job) { return *p.step >= p.jobs[job].stop; }
 
+// The solvent pair kernels' NEUT form is for the jobs of neutral solvent molecules,
+// the other for the rest: a batch that holds both kinds launches both, and each
+// leaves the other's jobs alone, so that a job's form (and bits) is its own.
+template <bool NEUT>
+__device__ __forceinline__ bool other_form(const SysPtrs& p, int32_t job) {
+    return (p.jobs[job].neutral != 0) != NEUT;
+}
+
 // Wave -> groups of the solvent pair kernels: the batch's sorted groups in
 // chunks of VV_CHUNK that never straddle two jobs (vv_chunk = first group, end,
 // job); a wave holds WAVE / NCHM consecutive groups of one chunk, so the job's
@@ -989,7 +997,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4
     // (uniform by construction; said once more after the early exits, or the job's
     // constants are taken for per-lane values and fill the vector registers)
     job = __builtin_amdgcn_readfirstlane(job);
-    if (held(p, job)) return;
+    if (held(p, job) || other_form<NEUT>(p, job)) return;
     double f[APS][3];
     double en[11];
 #pragma unroll
@@ -1075,7 +1083,7 @@ constexpr double FIX_MAX_L = 40.0;   // nm
 
 template <int APS, bool LJ00, bool VIR, int NCHM, bool NEUT>
 __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool valid, int chunk, int32_t job) {
-    if (held(p, job)) return;
+    if (held(p, job) || other_form<NEUT>(p, job)) return;
     double fi[APS][3];   // integers
     double ei[11];
 #pragma unroll
@@ -1408,7 +1416,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4
     int chunk = 0;
     if (!vv_wave<NCHM>(p, nwaves, k, valid, chunk, job)) return;
     job = __builtin_amdgcn_readfirstlane(job);   // uniform, as in k_vv
-    if (held(p, job)) return;
+    if (held(p, job) || other_form<NEUT>(p, job)) return;
     double f[APS][3];
     double en[11];
 #pragma unroll
@@ -3777,33 +3785,43 @@ static void launch_vv_near_aps(const SysPtrs& p, int32_t virial, int32_t neutral
     }
 #undef GAMD_NR_LAUNCH
 }
+// the batch's kinds of solvent molecules, a launch each: F(neutral, start, stop), the
+// timing events about the first and the last of them
+template <class F>
+static void each_form(int32_t form, hipEvent_t e0, hipEvent_t e1, F launch) {
+    const bool neut = (form & VV_NEUTRAL) != 0, chrg = (form & VV_CHARGED) != 0;
+    if (neut) launch(1, e0, chrg ? nullptr : e1);
+    if (chrg) launch(0, neut ? nullptr : e0, e1);
+}
 void launch_vv_near(const SysPtrs& p, int32_t aps, int32_t form, int32_t virial, hipStream_t s, hipEvent_t e0,
                     hipEvent_t e1) {
-    const int32_t neutral = (form & VV_NEUTRAL) ? 1 : 0;
-    switch (aps * 2 + ((form & VV_LJ00) ? 1 : 0)) {
-        case 2: launch_vv_near_aps<1, false>(p, virial, neutral, e0, e1, s); break;
-        case 3: launch_vv_near_aps<1, true>(p, virial, neutral, e0, e1, s); break;
-        case 4: launch_vv_near_aps<2, false>(p, virial, neutral, e0, e1, s); break;
-        case 5: launch_vv_near_aps<2, true>(p, virial, neutral, e0, e1, s); break;
-        case 8: launch_vv_near_aps<4, false>(p, virial, neutral, e0, e1, s); break;
-        case 9: launch_vv_near_aps<4, true>(p, virial, neutral, e0, e1, s); break;
-        case 7: launch_vv_near_aps<3, true>(p, virial, neutral, e0, e1, s); break;
-        default: launch_vv_near_aps<3, false>(p, virial, neutral, e0, e1, s); break;
-    }
+    each_form(form, e0, e1, [&](int32_t neutral, hipEvent_t a, hipEvent_t b) {
+        switch (aps * 2 + ((form & VV_LJ00) ? 1 : 0)) {
+            case 2: launch_vv_near_aps<1, false>(p, virial, neutral, a, b, s); break;
+            case 3: launch_vv_near_aps<1, true>(p, virial, neutral, a, b, s); break;
+            case 4: launch_vv_near_aps<2, false>(p, virial, neutral, a, b, s); break;
+            case 5: launch_vv_near_aps<2, true>(p, virial, neutral, a, b, s); break;
+            case 8: launch_vv_near_aps<4, false>(p, virial, neutral, a, b, s); break;
+            case 9: launch_vv_near_aps<4, true>(p, virial, neutral, a, b, s); break;
+            case 7: launch_vv_near_aps<3, true>(p, virial, neutral, a, b, s); break;
+            default: launch_vv_near_aps<3, false>(p, virial, neutral, a, b, s); break;
+        }
+    });
 }
 void launch_vv(const SysPtrs& p, int32_t ncg, int32_t aps, int32_t form, int32_t virial, int32_t mixed,
                int32_t lanes, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
-    const int32_t neutral = (form & VV_NEUTRAL) ? 1 : 0;
-    switch (aps * 2 + ((form & VV_LJ00) ? 1 : 0)) {
-        case 2: launch_vv_aps<1, false>(p, ncg, virial, mixed, neutral, lanes, e0, e1, s); break;
-        case 3: launch_vv_aps<1, true>(p, ncg, virial, mixed, neutral, lanes, e0, e1, s); break;
-        case 4: launch_vv_aps<2, false>(p, ncg, virial, mixed, neutral, lanes, e0, e1, s); break;
-        case 5: launch_vv_aps<2, true>(p, ncg, virial, mixed, neutral, lanes, e0, e1, s); break;
-        case 8: launch_vv_aps<4, false>(p, ncg, virial, mixed, neutral, lanes, e0, e1, s); break;
-        case 9: launch_vv_aps<4, true>(p, ncg, virial, mixed, neutral, lanes, e0, e1, s); break;
-        case 7: launch_vv_aps<3, true>(p, ncg, virial, mixed, neutral, lanes, e0, e1, s); break;
-        default: launch_vv_aps<3, false>(p, ncg, virial, mixed, neutral, lanes, e0, e1, s); break;
-    }
+    each_form(form, e0, e1, [&](int32_t neutral, hipEvent_t a, hipEvent_t b) {
+        switch (aps * 2 + ((form & VV_LJ00) ? 1 : 0)) {
+            case 2: launch_vv_aps<1, false>(p, ncg, virial, mixed, neutral, lanes, a, b, s); break;
+            case 3: launch_vv_aps<1, true>(p, ncg, virial, mixed, neutral, lanes, a, b, s); break;
+            case 4: launch_vv_aps<2, false>(p, ncg, virial, mixed, neutral, lanes, a, b, s); break;
+            case 5: launch_vv_aps<2, true>(p, ncg, virial, mixed, neutral, lanes, a, b, s); break;
+            case 8: launch_vv_aps<4, false>(p, ncg, virial, mixed, neutral, lanes, a, b, s); break;
+            case 9: launch_vv_aps<4, true>(p, ncg, virial, mixed, neutral, lanes, a, b, s); break;
+            case 7: launch_vv_aps<3, true>(p, ncg, virial, mixed, neutral, lanes, a, b, s); break;
+            default: launch_vv_aps<3, false>(p, ncg, virial, mixed, neutral, lanes, a, b, s); break;
+        }
+    });
 }
 void launch_gen(const SysPtrs& p, int32_t npad, bool lng, int32_t virial, int32_t mixed, int32_t ngsol,
                 hipStream_t s, int32_t part) {

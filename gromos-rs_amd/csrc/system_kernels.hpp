@@ -153,10 +153,11 @@ void launch_job_pairs(const SysPtrs& p, int32_t njobs, hipStream_t s);
 // capacities = counts; 2: the previous counts without slack (test hook)
 void launch_caps(const SysPtrs& p, int32_t ncg, int32_t mode, hipStream_t s);
 void launch_gather(const SysPtrs& p, int32_t npad, int32_t mixed, hipStream_t s);
-// form: VV_LJ00 (LJ on the first-first atom pair only) | VV_NEUTRAL (neutral
-// solvent molecules: the mixed kernel sums the RF polynomial per molecule pair);
+// form: VV_LJ00 (LJ on the first-first atom pair only) | VV_NEUTRAL (the batch has
+// jobs of neutral solvent molecules, whose RF polynomial is summed per molecule
+// pair) | VV_CHARGED (it has other jobs); JobDev::neutral tells a job's kind;
 // lanes: lanes per solvent molecule (4, 8 or 16)
-constexpr int32_t VV_LJ00 = 1, VV_NEUTRAL = 2;
+constexpr int32_t VV_LJ00 = 1, VV_NEUTRAL = 2, VV_CHARGED = 4;
 constexpr int32_t NXCD_SCHED = 9;   // the persistent far-pair kernel's counters: one per XCD, waves done
 void launch_vv(const SysPtrs& p, int32_t ncg, int32_t aps, int32_t form, int32_t virial, int32_t mixed,
                int32_t lanes, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
