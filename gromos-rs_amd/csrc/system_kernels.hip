@@ -150,9 +150,15 @@ __global__ void __launch_bounds__(BLOCK) k_cell_order(SysPtrs p, int32_t ncell) 
 //               boxes), so that a difference of two wraps to the nearest image by
 //               itself; bit patterns of integers
 //   atoms 1..   FP32 offsets from the first atom (difference taken in FP64)
-//   w           the molecule's dipole sum q x, a component in each of atoms 0-2
+//   w           the molecule's dipole sum q x, a component in each of atoms 0-2; NaN
+//               in atom 0's where a coordinate of the first atom is not finite (a
+//               fraction cannot say so; the other sites' offsets do)
+__device__ __forceinline__ float not_finite(d3 x) {   // 0, or NaN
+    return (float)((x.x - x.x) + (x.y - x.y) + (x.z - x.z));
+}
 __device__ __forceinline__ float4 far_copy(const Box& b, int j, d3 x0, d3 x, float w) {
     if (j > 0) return make_float4((float)(x.x - x0.x), (float)(x.y - x0.y), (float)(x.z - x0.z), w);
+    w += not_finite(x);
     if (b.kind != 1) return make_float4(0.f, 0.f, 0.f, w);
     return make_float4(box_fraction(x.x, b.invL[0]), box_fraction(x.y, b.invL[1]), box_fraction(x.z, b.invL[2]), w);
 }
@@ -1126,6 +1132,7 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
         const float c6_00 = uniform((float)J.sv_c6[0]), c12_00 = uniform((float)J.sv_c12[0]);
         int32_t ax, ay, az;
         float mua[3];   // NEUT: own dipole
+        float lost;     // one-site molecules: NaN where the position is not finite
         {
             const float4 a0 = p.xf[sk];
             ax = __float_as_int(a0.x);
@@ -1134,6 +1141,7 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
             dax[0] = day[0] = daz[0] = 0.f;
             mua[0] = APS >= 3 ? a0.w : 0.f;
             mua[1] = mua[2] = 0.f;
+            lost = a0.w;
 #pragma unroll
             for (int i = 1; i < APS; ++i) {
                 const float4 a = p.xf[sk + i];
@@ -1199,6 +1207,7 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
                         sx = fmaf(ix, uh[0], ix * ul[0]);
                         sy = fmaf(iy, uh[1], iy * ul[1]);
                         sz = fmaf(iz, uh[2], iz * ul[2]);
+                        if (APS == 1) sx += lost + r0.w;   // 0, or NaN
                     } else {
                         shift32(J.box, xyz(p.xq[sk]), xyz(p.xq[sm]), sx, sy, sz);
                     }
@@ -3441,7 +3450,7 @@ __global__ void __launch_bounds__(BLOCK) k_integrate(SysPtrs p, int32_t ncg, int
         if (MIXED && write_xq && !solute_group) {
             // the dipole is known after the last atom
             const int32_t a = p.o2s[s];
-            p.xf[a].w = (float)mu.x;
+            p.xf[a].w = (float)mu.x + not_finite(d3{x_first.x, x_first.y, x_first.z});
             if (n > 1) p.xf[a + 1].w = (float)mu.y;
             if (n > 2) p.xf[a + 2].w = (float)mu.z;
         }
