@@ -102,6 +102,7 @@ __global__ void k_scatter(SysPtrs p, int32_t ncg) {
 
 // a coordinate's place in the box as 32-bit fixed point (the bits of an integer):
 // the difference of two wraps to the nearest image by itself
+constexpr int32_t FIX_LOST = INT32_MIN;   // s_fix w: the point is not finite (no fraction says so)
 __device__ __forceinline__ float box_fraction(double x, double invL) {
     double u = x * invL;
     u -= floor(u);
@@ -125,6 +126,9 @@ __global__ void __launch_bounds__(BLOCK) k_cell_order(SysPtrs p, int32_t ncell) 
             f.x = __float_as_int(box_fraction(p.ref[3 * c], b.invL[0]));
             f.y = __float_as_int(box_fraction(p.ref[3 * c + 1], b.invL[1]));
             f.z = __float_as_int(box_fraction(p.ref[3 * c + 2], b.invL[2]));
+            const double lost = (p.ref[3 * c] - p.ref[3 * c]) + (p.ref[3 * c + 1] - p.ref[3 * c + 1]) +
+                                (p.ref[3 * c + 2] - p.ref[3 * c + 2]);   // 0, or NaN
+            if (!(lost == 0.0)) f.w |= FIX_LOST;
         }
         p.s_fix[k] = f;
     };
@@ -224,7 +228,9 @@ __device__ __forceinline__ double ref_d2(const Box& b, d3 lo, d3 hi) {
 // (nim_search), so the pair set is the reference's to the bit.  The near / far
 // classification needs no such care: either kernel may take a pair.
 // A distance that is not a number is a pair, as in the reference, and a near one: the
-// FP64 path lists every partner as near and reads its slots from the start only.
+// FP64 path lists every partner as near and reads its slots from the start only.  (In
+// a rectangular box a point that is not finite is marked, and distances that may
+// involve one are all taken the reference's way.)
 // Bound by instructions: about 60 vector ones per 64 candidates.  32,768 waters at
 // 1.4 nm: 109 us (156 with FP64 distances and every group's cursors in vector
 // registers); 128 x 4,000 waters at 1.2 nm: 1,041 us (1,544).
@@ -288,6 +294,7 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
     // uniform address in the candidate loop: a broadcast through LDS instead of
     // lane reads on the vector ALU
     __shared__ int4 s_own[NBL_WAVES][WAVE];
+    __shared__ int32_t s_lost;         // a candidate so far has no place (FIX_LOST)
     const int32_t c = xcd_block(ncell);
     if (c < 0) return;
     const int32_t s0 = p.cell_start[c], s1 = p.cell_start[c + 1];
@@ -301,6 +308,7 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
     const int32_t nx = J.ncell[0], ny = J.ncell[1], nz = J.ncell[2];
     const int32_t local = c - J.cell_off;
     const int32_t cc[3] = {local % nx, (local / nx) % ny, local / (nx * ny)};
+    if (threadIdx.x == 0) s_lost = 0;
     // the stencil as x runs of sorted groups, in (z, y, x-segment) order
     if (wv == 0) {
         const int32_t nyy = ny >= 2 * CELL_R + 1 ? 2 * CELL_R + 1 : ny;
@@ -361,7 +369,9 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
         const int32_t gi = wv + NBL_WAVES * lane;
         const bool own = gi < nr;
         const int32_t k = own ? rb + gi : rb;
-        const int4 kf = p.s_fix[k];
+        int4 kf = p.s_fix[k];
+        const uint64_t lost_mask = RECT ? __ballot(kf.w < 0) : 0ull;
+        kf.w &= ~FIX_LOST;
         const int32_t ck = kf.w, nk = p.s_cg_n[k];
         const uint64_t own_mask = __ballot(own);
         const int32_t n_own = (int32_t)__popcll(own_mask);   // a prefix of the lanes
@@ -390,13 +400,17 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
                     if (run_off[mid] <= g) lo = mid; else hi = mid - 1;
                 }
                 const int32_t m = run_m0[lo] + (g - run_off[lo]);
-                sfix[q] = p.s_fix[m];
+                int4 mf = p.s_fix[m];
+                if (RECT && mf.w < 0) s_lost = 1;
+                mf.w &= ~FIX_LOST;
+                sfix[q] = mf;
                 sm[q] = m;
                 sst[q] = p.s_cg_start[m];
                 snn[q] = p.s_cg_n[m];
             }
             __syncthreads();
             if (!own_mask) continue;   // wave-uniform; the barriers above are reached by all
+            const bool lost_piece = RECT && __builtin_amdgcn_readfirstlane(s_lost) != 0;
             // a group at a time over the piece: its data and its slot's cursors sit in
             // scalar registers, the candidates come from LDS for each group again
             // (the wave's own groups are lanes 0 .. n_own - 1: gi = wv + 4 lane < nr)
@@ -406,6 +420,7 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
                 const int32_t ox = __builtin_amdgcn_readfirstlane(ov.x), oy = __builtin_amdgcn_readfirstlane(ov.y),
                               oz = __builtin_amdgcn_readfirstlane(ov.z), ck_t = __builtin_amdgcn_readfirstlane(ov.w);
                 const bool sol_k = (solk_mask >> t) & 1ull;
+                const float tol = lost_piece || ((lost_mask >> t) & 1ull) ? INFINITY : tol_l;
                 const int32_t vbase = bcast(vv_base, t), vcap = bcast(vv_end, t) - vbase;
                 int32_t vlo = vbase + bcast(vv_nn, t), vhi = vbase + vcap - 1 - bcast(vv_nf, t);
                 int32_t ns = bcast(gen_ns, t), nl = bcast(gen_nl, t);
@@ -424,13 +439,14 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
                         in = !(d2f > c2lf);
                         lng = d2f > c2sf;
                         near = d2f < nearf;
-                        bool doubt = fabsf(d2f - c2lf) <= tol_l;
+                        bool doubt = fabsf(d2f - c2lf) <= tol;
                         if (twin) doubt = doubt || fabsf(d2f - c2sf) <= tol_s;
                         if (__builtin_expect(doubt, 0)) {
                             const d3 r = nim_rect(box, ld3(p.s_ref, i), ld3(p.s_ref, sm[qq]));
                             const double d2 = r.x * r.x + r.y * r.y + r.z * r.z;
                             in = !(d2 > c2l);
                             lng = d2 > c2s;
+                            near = !(d2 >= near_r2);
                         }
                     } else {
                         const d3 r = nim_search(box, ld3(p.s_ref, i), ld3(p.s_ref, sm[qq]));

@@ -49,6 +49,7 @@ struct SysPtrs {
     int32_t pert_twin;             // ... in a job with a twin range
     int32_t any_rect, any_other;   // the batch holds jobs with a rectangular / another boundary
     int4* s_fix;               // per sorted group: reference point as box fractions (k_nbl), original group
+                               // (sign bit: the point is not finite)
     int32_t* s2o;
     int32_t* s_atom_cg;
     int32_t* s_type;

@@ -83,3 +83,24 @@ def test_non_finite_point_in_a_one_cell_box(prec, boundary):
         assert not np.any(np.abs(f).max(axis=-1).reshape(-1, 3).max(axis=-1) < 1e6)
         assert len(ds.pairlist()["solvent_short"]) >= n
     ds.close()
+
+
+@pytest.mark.parametrize("prec", [rt.FP64, rt.MIXED])
+@pytest.mark.parametrize("side", [0, 1])
+def test_non_finite_reference_point_is_listed(prec, side):
+    """a molecule without a place on x (the comparison with the cutoff fails, as in the reference): it has the
+    molecules in reach of its cell as partners, whichever of the two comes first, and their forces show it"""
+    s = gen.spc_water_box(3, box=4.0, seed=2, rcutp=0.9, rcutl=0.9, temperature=0.0)
+    first = np.array([[2.2, 2.2, 2.2], [1.1, 0.2, 0.2], [0.1, 0.2, 0.2]])
+    lost = 2 if side else 0
+    if not side:
+        first = first[::-1].copy()
+    place(s, first)
+    s.pos[3 * lost:3 * lost + 3, 0] = np.nan
+    ds = rt.DeviceSystem(s, precision=prec, use_settle=False)
+    for _ in range(2):   # the first build, and one into slots sized from it
+        ds.set_state(s.pos)
+        f = ds.forcefield_apply()["forces"].reshape(3, 3, 3)
+        assert not np.any(np.abs(f[1]).max(axis=-1) < 1e6)
+        assert not np.any(np.abs(f[lost]).max(axis=-1) < 1e6)
+    ds.close()
