@@ -1160,7 +1160,8 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
             lost = a0.w;
 #pragma unroll
             for (int i = 1; i < APS; ++i) {
-                const float4 a = p.xf[sk + i];
+                // (a solute group has no entries, and its next atoms are not its own)
+                const float4 a = n > 0 ? p.xf[sk + i] : make_float4(0.f, 0.f, 0.f, 0.f);
                 dax[i] = a.x;
                 day[i] = a.y;
                 daz[i] = a.z;
