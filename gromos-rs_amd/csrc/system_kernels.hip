@@ -697,6 +697,11 @@ __device__ __forceinline__ float uniform(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
+__device__ __forceinline__ double uniform(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
 // nearest-image vector between two group first atoms in FP64, returned as
 // float, with the reference's image choice (ties included)
 __device__ __forceinline__ void shift32(const Box& b, d3 A, d3 B, float& x, float& y, float& z) {
@@ -1085,20 +1090,26 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4
 // The nearest image: in a rectangular box wider than twice the list cutoff the
 // first atoms' box fractions are subtracted as 32-bit integers, whose wrap is the
 // nearest image (12 operations against 24 in FP64; a coordinate is held to L / 2^33,
-// 1.2e-9 nm at 10 nm, a fortieth of the FP32 rounding of r, and boxes over FIX_MAX_L
-// keep the other form).  Listed pairs there are never at the half-box tie.  Other boxes take shift32 in FP64.
+// 1.2e-9 nm at 10 nm, a fortieth of the FP32 rounding of r; scaled in FP64 and rounded
+// to FP32 once, as the other form's vector).  Listed pairs there are never at the
+// half-box tie.  Other boxes, and those over FIX_MAX_L, take shift32 in FP64.
 //
-// Fixed point: groups of VV_GROUP entries are summed in FP32 (every partner here
-// is beyond the near radius, so the terms are moderate), and each group's sums
-// are rounded to integers, which FP64 adds exactly (below 2^53), so the result
-// depends neither on the lane count nor on the order.  A group takes every
-// VV_SPREAD-th entry of a run of VV_SPREAD x VV_GROUP, so that neighbouring lanes
-// read neighbouring entries, whose molecules are near each other in memory.
+// Sums: forces of VV_GROUP entries in FP32 (every partner here is beyond the near
+// radius, so the terms are moderate), energies per molecule pair and then over
+// the group, dipole products and the virial's R (x) F in FP64.  These are rounded to
+// integers, which FP64 adds exactly (below 2^53), so the result depends neither on
+// the lane count nor on the order.  A group takes every VV_SPREAD-th entry of a run
+// of VV_SPREAD x VV_GROUP, so that neighbouring lanes read neighbouring entries,
+// whose molecules are near each other in memory.  Error against FP64 over 150 boxes
+// of 1,000 waters: forces 1.737e-4 kJ/mol/nm RMS, E_crf 1.91e-3 kJ/mol, virial
+// 1.68e-3 (standard deviations); with FP64 image vectors, energies over nine atom
+// pairs and the virial in FP64 over pairs 1.780e-4, 1.95e-3, 1.75e-3; energies in one
+// FP32 chain over the group's pairs, the virial in FP32 too, 1.738e-4, 2.33e-3, 1.72e-3.
 //
-// VALU bound (about 225 instruction slots per entry, reciprocal square roots
-// counting four; four waves per SIMD).  32,768 waters at 1.4 nm: 72 us (101 with
+// VALU bound (about 230 instruction slots per entry, reciprocal square roots
+// counting four; four waves per SIMD).  32,768 waters at 1.4 nm: 77 us (101 with
 // FP64 shifts, the job's constants in vector registers, int64 sums per group and
-// energies of the canonical side only); 128 x 4,000 waters at 1.2 nm: 697 us
+// energies of the canonical side only); 128 x 4,000 waters at 1.2 nm: 721 us
 // (1,077); 2,187 waters at 1.2 nm with the virial: 21 us (37).
 constexpr int VV_SPREAD = 16;        // a multiple of every lane count
 constexpr double FIX_MAX_L = 40.0;   // nm
@@ -1130,15 +1141,10 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
         const bool fix = __builtin_amdgcn_readfirstlane(
             J.box.kind == 1 && fmin(J.box.L[0], fmin(J.box.L[1], J.box.L[2])) > 4.0 * J.cell_min &&
             fmax(J.box.L[0], fmax(J.box.L[1], J.box.L[2])) < FIX_MAX_L);
-        // the fixed-point unit L / 2^32 in two parts: one float would scale every
-        // distance by the same rounding, up to 6e-8
-        float uh[3], ul[3];
+        // the fixed-point unit L / 2^32
+        double un[3];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const double u = J.box.L[c] * (1.0 / 4294967296.0);
-            uh[c] = uniform((float)u);
-            ul[c] = uniform((float)(u - (double)uh[c]));
-        }
+        for (int c = 0; c < 3; ++c) un[c] = uniform(J.box.L[c] * (1.0 / 4294967296.0));
         const float c2 = (float)J.crf.crf_2cut3i, cc = (float)J.crf.crf_cut, c3 = (float)J.crf.crf_cut3i;
         float qq[APS][APS];
 #pragma unroll
@@ -1147,16 +1153,13 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
             for (int j = 0; j < APS; ++j) qq[i][j] = uniform((float)J.sv_qq[i * 4 + j]);
         const float c6_00 = uniform((float)J.sv_c6[0]), c12_00 = uniform((float)J.sv_c12[0]);
         int32_t ax, ay, az;
-        float mua[3];   // NEUT: own dipole
-        float lost;     // one-site molecules: NaN where the position is not finite
+        float lost;   // one-site molecules: NaN where the position is not finite
         {
             const float4 a0 = p.xf[sk];
             ax = __float_as_int(a0.x);
             ay = __float_as_int(a0.y);
             az = __float_as_int(a0.z);
             dax[0] = day[0] = daz[0] = 0.f;
-            mua[0] = APS >= 3 ? a0.w : 0.f;
-            mua[1] = mua[2] = 0.f;
             lost = a0.w;
 #pragma unroll
             for (int i = 1; i < APS; ++i) {
@@ -1165,26 +1168,17 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
                 dax[i] = a.x;
                 day[i] = a.y;
                 daz[i] = a.z;
-                if (APS >= 3 && i < 3) mua[i] = a.w;
-            }
-            if (APS == 2) {
-                const float q1 = (float)J.sv_q[1];
-                mua[0] = q1 * dax[APS - 1];
-                mua[1] = q1 * day[APS - 1];
-                mua[2] = q1 * daz[APS - 1];
             }
         }
         uint32_t next = chunk < n ? p.vv_ent[ef + chunk] : 0u;
         for (int32_t b0 = 0; __any(b0 < n); b0 += VV_SPREAD * VV_GROUP) {
 #pragma unroll 1
             for (int32_t g = 0; g < VV_SPREAD; g += NCHM) {
-                float fs[APS][3], w[9];
+                float fs[APS][3];
 #pragma unroll
                 for (int i = 0; i < APS; ++i) fs[i][0] = fs[i][1] = fs[i][2] = 0.f;
-#pragma unroll
-                for (int c = 0; c < 9; ++c) w[c] = 0.f;
                 float msx = 0.f, msy = 0.f, msz = 0.f;   // NEUT: sum of partner dipoles
-                float el = 0.f, ec = 0.f;
+                float els = 0.f, ecs = 0.f;
                 int32_t x = b0 + g + chunk;
 #pragma unroll 1
                 for (int t = 0; t < VV_GROUP; ++t) {
@@ -1218,12 +1212,10 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
                     }
                     float sx, sy, sz;
                     if (fix) {
-                        const float ix = (float)(int32_t)((uint32_t)ax - __float_as_uint(r0.x)),
-                                    iy = (float)(int32_t)((uint32_t)ay - __float_as_uint(r0.y)),
-                                    iz = (float)(int32_t)((uint32_t)az - __float_as_uint(r0.z));
-                        sx = fmaf(ix, uh[0], ix * ul[0]);
-                        sy = fmaf(iy, uh[1], iy * ul[1]);
-                        sz = fmaf(iz, uh[2], iz * ul[2]);
+                        // exact in FP64, rounded to FP32 once, as shift32's
+                        sx = (float)((double)(int32_t)((uint32_t)ax - __float_as_uint(r0.x)) * un[0]);
+                        sy = (float)((double)(int32_t)((uint32_t)ay - __float_as_uint(r0.y)) * un[1]);
+                        sz = (float)((double)(int32_t)((uint32_t)az - __float_as_uint(r0.z)) * un[2]);
                         if (APS == 1) sx += lost + r0.w;   // 0, or NaN
                     } else {
                         shift32(J.box, xyz(p.xq[sk]), xyz(p.xq[sm]), sx, sy, sz);
@@ -1234,6 +1226,7 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
                         msz += mz;
                     }
                     float F[3] = {0.f, 0.f, 0.f};
+                    float el = 0.f, ec = 0.f;   // this molecule pair's
 #pragma unroll
                     for (int i = 0; i < APS; ++i) {
                         const float cx = i ? sx + dax[i] : sx, cy = i ? sy + day[i] : sy, cz = i ? sz + daz[i] : sz;
@@ -1292,20 +1285,29 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
                         fs[i][1] = gy;
                         fs[i][2] = gz;
                     }
-                    if (VIR) {   // R (x) F; the rest comes from the forces at the end (vv64_lane)
+                    els += el;
+                    ecs += ec;
+                    if (VIR) {   // R (x) F, to integers at once (nine FP64 sums fewer in registers,
+                                 // which spill); the rest comes from the forces at the end (vv64_lane)
+                        const double R[3] = {(double)sx * EX_SCALE, (double)sy * EX_SCALE, (double)sz * EX_SCALE};
 #pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            w[c] = fmaf(sx, F[c], w[c]);
-                            w[3 + c] = fmaf(sy, F[c], w[3 + c]);
-                            w[6 + c] = fmaf(sz, F[c], w[6 + c]);
-                        }
+                        for (int c = 0; c < 3; ++c)
+#pragma unroll
+                            for (int x = 0; x < 3; ++x) ei[2 + 3 * x + c] += rint(R[x] * (double)F[c]);
                     }
                 }
-                double en[2] = {(double)el, (double)ec};
+                double en[2] = {(double)els, (double)ecs};
                 const double ms[3] = {(double)msx, (double)msy, (double)msz};
-                if (NEUT && APS > 1)
-                    en[1] = fma(2.0 * J.crf.crf_2cut3i * J.fpepsi,
-                                fma((double)mua[0], ms[0], fma((double)mua[1], ms[1], (double)mua[2] * ms[2])), en[1]);
+                if (NEUT && APS > 1) {
+                    double mu[3] = {0.0, 0.0, 0.0};   // own dipole
+#pragma unroll
+                    for (int i = 1; i < APS; ++i) {
+                        mu[0] = fma(J.sv_q[i], (double)dax[i], mu[0]);
+                        mu[1] = fma(J.sv_q[i], (double)day[i], mu[1]);
+                        mu[2] = fma(J.sv_q[i], (double)daz[i], mu[2]);
+                    }
+                    en[1] = fma(2.0 * J.crf.crf_2cut3i * J.fpepsi, fma(mu[0], ms[0], fma(mu[1], ms[1], mu[2] * ms[2])), en[1]);
+                }
 #pragma unroll
                 for (int i = 0; i < APS; ++i) {
                     const double kf = -J.sv_q[i] * J.fpepsi * J.crf.crf_cut3i;
@@ -1318,9 +1320,6 @@ __device__ __forceinline__ void vv_mx_wave(const SysPtrs& p, int32_t k, bool val
                 }
                 ei[0] += rint(en[0] * EX_SCALE);
                 ei[1] += rint(en[1] * EX_SCALE);
-                if (VIR)
-#pragma unroll
-                    for (int c = 0; c < 9; ++c) ei[2 + c] += rint((double)w[c] * EX_SCALE);
             }
         }
     }
