@@ -240,15 +240,15 @@ struct gromos_amd_bonded_plan {
     int32_t nterms = 0;
     int4* atoms = nullptr;
     double4* prm = nullptr;
-    int32_t* kind = nullptr;
-    double* tf = nullptr;
-    double* part = nullptr;      // BD_SUMS per block of terms
-    uint32_t* done = nullptr;    // blocks that have written theirs
+    int32_t* kind = nullptr;     // nterms, then the count of blocks done (uploaded as zero)
+    double* tf = nullptr;        // 12 per term, then BD_SUMS per block of terms
     int32_t* aoff = nullptr;
     int32_t* aref = nullptr;
     int32_t n[4] = {0, 0, 0, 0};
+    double* part() const { return tf + 12 * (size_t)nterms; }
+    uint32_t* done() const { return (uint32_t*)(kind + nterms); }
     ~gromos_amd_bonded_plan() {
-        for (void* p : {(void*)atoms, (void*)prm, (void*)kind, (void*)tf, (void*)part, (void*)done, (void*)aoff, (void*)aref})
+        for (void* p : {(void*)atoms, (void*)prm, (void*)kind, (void*)tf, (void*)aoff, (void*)aref})
             if (p) (void)hipFree(p);
     }
 };
@@ -279,13 +279,13 @@ extern "C" int gromos_amd_bonded_plan_create(const gromos_amd_bonded* b, gromos_
     std::memcpy(P->n, t.n, sizeof P->n);
     int rc = dev_copy(P->atoms, t.atoms);
     rc = rc ? rc : dev_copy(P->prm, t.prm);
+    t.kind.push_back(0);
     rc = rc ? rc : dev_copy(P->kind, t.kind);
     rc = rc ? rc : dev_copy(P->aoff, aoff);
     rc = rc ? rc : dev_copy(P->aref, aref);
-    if (!rc && hipMalloc(&P->tf, std::max<size_t>(P->nterms, 1) * 12 * sizeof(double)) != hipSuccess)
+    const size_t scratch = 12 * (size_t)P->nterms + BD_SUMS * (size_t)term_blocks(P->nterms);
+    if (!rc && hipMalloc(&P->tf, scratch * sizeof(double)) != hipSuccess)
         rc = fail(GROMOS_AMD_ENOMEM, "bonded_plan_create: device memory");
-    rc = rc ? rc : dev_copy(P->part, std::vector<double>(BD_SUMS * (size_t)term_blocks(P->nterms)));
-    rc = rc ? rc : dev_copy(P->done, std::vector<uint32_t>(1, 0u));
     if (rc) {
         delete P;
         return rc;
@@ -317,7 +317,7 @@ extern "C" int gromos_amd_bonded_forces(const gromos_amd_bonded_plan* p, const d
     bd.fb = forces;
     bd.nterms = p->nterms;
     bd.natoms = p->n_atoms;
-    k_bd_terms_sum<<<term_blocks(bd.nterms), BD_BLOCK, 0, s>>>(bd, pos, p->part, p->done, out);
+    k_bd_terms_sum<<<term_blocks(bd.nterms), BD_BLOCK, 0, s>>>(bd, pos, p->part(), p->done(), out);
     launch_bonded_gather(bd, s);
     HIPCHK(hipGetLastError());
     return 0;
