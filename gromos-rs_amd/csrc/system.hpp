@@ -80,10 +80,9 @@ struct JobDev {
     int32_t bd_n[4];                       // terms per kind: bonds, angles, dihedrals, impropers
 };
 
-// energy partial rows: per kernel slot and block, 12 doubles
-// (e_lj, e_crf, vir[9], extra)
+// energy partial rows: the excluded / 1-4 / self terms' per block of atoms, and the
+// solute atoms' records, 12 doubles (e_lj, e_crf, vir[9], dH/dlambda)
 constexpr int ROW = 12;
-enum Slot { SLOT_VV = 0, SLOT_GEN = 1, SLOT_LONG = 2, SLOT_EXCL = 3, SLOT_KIN = 4, NSLOT = 5 };
 
 // a force component at or beyond this (kJ mol^-1 nm^-1), or a non-finite one,
 // marks its job as diverged (the fixed-point conversions saturate at twice it)

@@ -95,7 +95,7 @@ void rebox_image(JobImage& im, const Box& box) {
 // device bytes per padded atom / per charge group held by a batch (the arrays
 // of gromos_amd_system), used for admission by footprint
 constexpr int64_t BYTES_PER_ATOM = 2 * 2 * 24 + 7 * 24 + 32 + 16 + 8 + 4 + 8 + 8 + 4 + 12 + 16 + 41 +
-                                   NSLOT * ROW * 8 * 4 / BLOCK + 16;
+                                   ROW * 8 / BLOCK + 1 + 16;
 constexpr int64_t BYTES_PER_CG = 2 * 24 + 16 + 16 + 16 + 4 * 8 + 2 * 8 + 2 * 4 + 8;
 
 // setup_lincs (constraints.rs:1168-1220): sd[k] = 1 / sqrt(1/m_i + 1/m_j); two
@@ -677,7 +677,7 @@ int layout_batch(gromos_amd_system* S, const std::vector<const JobImage*>& imgs,
     S->ncg = (int32_t)ncg;
     S->ncell = (int32_t)cell_off;
     S->nmol = (int32_t)mol_first.size();
-    S->nrow_blocks = (int32_t)(align_up(npad * 4, BLOCK) / BLOCK);   // 4 lanes per atom in the pair kernel
+    S->nrow_blocks = (int32_t)(npad / BLOCK);
     S->nsnb = std::max(1, I0.P.nsnb);
     S->use_settle = use_settle;
     S->do_virial = do_virial || any_baro;   // the pressure needs every step's virial
@@ -912,7 +912,7 @@ int layout_batch(gromos_amd_system* S, const std::vector<const JobImage*>& imgs,
         (rc = S->reserve(S->d_f_x, n3, true)) ||
         (rc = S->reserve(S->d_xf, npa, true)) || (rc = S->reserve(S->d_fi_s, n3, true)) ||
         (rc = S->reserve(S->d_fi_long_s, n3, true)) ||
-        (rc = S->reserve(S->d_rows, (size_t)NSLOT * S->nrow_blocks * ROW, true)) ||
+        (rc = S->reserve(S->d_rows, (size_t)S->nrow_blocks * ROW, true)) ||
         (rc = S->reserve(S->d_settle_fail, (size_t)njobs, true)) ||
         (rc = S->reserve(S->d_force_fail, (size_t)njobs, true)) ||
         (rc = S->reserve(S->d_therm_scale, (size_t)njobs, true)) ||
@@ -965,7 +965,7 @@ int layout_batch(gromos_amd_system* S, const std::vector<const JobImage*>& imgs,
     HIPCHK(hipMemsetAsync(S->d_fi_near, 0, n3 * sizeof(long long), st));   // padding slots stay zero
     HIPCHK(hipMemsetAsync(S->d_step, 0, sizeof(int32_t), st));
     HIPCHK(hipMemsetAsync(S->d_step_done, 0, sizeof(uint32_t), st));
-    HIPCHK(hipMemsetAsync(S->d_rows, 0, (size_t)NSLOT * S->nrow_blocks * ROW * sizeof(double), st));
+    HIPCHK(hipMemsetAsync(S->d_rows, 0, (size_t)S->nrow_blocks * ROW * sizeof(double), st));
     HIPCHK(hipMemsetAsync(S->d_fi_long_s, 0, n3 * sizeof(long long), st));
     HIPCHK(hipMemsetAsync(S->d_s_cg_n, 0, (nc + 1) * sizeof(int32_t), st));
     HIPCHK(hipMemsetAsync(S->d_vv_cnt, 0, (nc + 1) * sizeof(int64_t), st));
@@ -1290,7 +1290,7 @@ int forcefield(gromos_amd_system* S, bool assemble) {
             HIPCHK(hipEventRecord(S->ev_fork, st));
             HIPCHK(hipStreamWaitEvent(S->side, S->ev_fork, 0));
             launch_vv_near(p, aps, form, S->do_virial, S->side, na, nb);
-            launch_gen(p, npad, false, S->do_virial, mixed, 0, S->side, GEN_SOLUTE);
+            launch_gen(p, false, S->do_virial, mixed, 0, S->side, GEN_SOLUTE);
             launch_excl14(p, npad, 0, S->d_excl_blocks, S->n_excl_blocks, S->side);
             launch_bonded(p.bd, p.x_cur, S->side);
             HIPCHK(hipEventRecord(S->ev_join, S->side));
@@ -1316,10 +1316,10 @@ int forcefield(gromos_amd_system* S, bool assemble) {
         S->timed_pairs += active_pairs(S, 2) / 2 * (int64_t)aps * aps;
     }
     const int32_t ngsol = (int32_t)S->host_counters[4];
-    launch_gen(p, npad, false, S->do_virial, mixed, ngsol, st, split ? GEN_SOLVENT : GEN_ALL);
+    launch_gen(p, false, S->do_virial, mixed, ngsol, st, split ? GEN_SOLVENT : GEN_ALL);
     S->pair_count += active_pairs(S, 0);
     if (S->twin && (rebuild || !S->long_computed)) {
-        launch_gen(p, npad, true, 1, mixed, ngsol, st);
+        launch_gen(p, true, 1, mixed, ngsol, st);
         S->long_computed = true;
         S->pair_count += active_pairs(S, 1);
     }
@@ -1357,7 +1357,7 @@ static int launch_step_graph(gromos_amd_system* S) {
         HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         launch_vv(p, S->ncg, aps, form, S->do_virial, mixed, S->vv_lanes, st);
         if (mixed) launch_vv_near(p, aps, form, S->do_virial, st);
-        launch_gen(p, S->npad, false, S->do_virial, mixed, (int32_t)S->host_counters[4], st);
+        launch_gen(p, false, S->do_virial, mixed, (int32_t)S->host_counters[4], st);
         launch_excl14(p, S->npad, 0, S->d_excl_blocks, S->n_excl_blocks, st);
         launch_bonded(p.bd, p.x_cur, st);
         launch_integrate(p, S->ncg, S->twin ? 1 : 0, 1, mixed, st);
@@ -1662,7 +1662,6 @@ SysPtrs gromos_amd_system::ptrs() const {
     p.xf = d_xf;
     p.fi_s = d_fi_s;
     p.fi_long_s = d_fi_long_s;
-    p.nrow_blocks = nrow_blocks;
     p.f_s = d_f_s;
     p.f_long_s = d_f_long_s;
     p.f_x = d_f_x;

@@ -647,14 +647,11 @@ __device__ __forceinline__ void add_virial(double (&v)[ROW], d3 r, double fx, do
     v[8] += r.z * fx; v[9] += r.z * fy; v[10] += r.z * fz;
 }
 
-__device__ __forceinline__ void write_row(double (&v)[ROW], double* rows, int slot, int nblocks, int32_t blk) {
+__device__ __forceinline__ void write_row(double (&v)[ROW], double* rows, int32_t blk) {
     __shared__ double lds[17 * ROW];
     block_sum<ROW>(v, lds);
     if (threadIdx.x < ROW)
-        rows[((int64_t)slot * nblocks + blk) * ROW + threadIdx.x] = lds[16 * ROW + threadIdx.x];
-}
-__device__ __forceinline__ void write_row(double (&v)[ROW], double* rows, int slot, int nblocks) {
-    write_row(v, rows, slot, nblocks, (int32_t)blockIdx.x);
+        rows[(int64_t)blk * ROW + threadIdx.x] = lds[16 * ROW + threadIdx.x];
 }
 
 // ---- mixed precision: FP32 pair arithmetic, FP64 per-lane partial sums,
@@ -2532,7 +2529,7 @@ __global__ void __launch_bounds__(BLOCK) k_excl14(SysPtrs p, int32_t npad, int32
         p.f_x[3 * i + 1] = fy;
         p.f_x[3 * i + 2] = fz;
     }
-    write_row(v, p.rows, SLOT_EXCL, p.nrow_blocks, blk);
+    write_row(v, p.rows, blk);
 }
 
 // total force on each original atom
@@ -3547,8 +3544,8 @@ __global__ void __launch_bounds__(BLOCK) k_vv_parts(SysPtrs p, int32_t with_viri
 }
 
 // One block per job: sums the job's partial rows in a fixed order and writes
-// the step record (e_lj, e_crf, e_pot, e_kin, dhdl, vir[9]).  Column 11 of a
-// row is E_kin in the kinetic slot and dH/dlambda in the others.
+// the step record (e_lj, e_crf, e_pot, e_kin, dhdl, vir[9], covalent energies).
+// Column 11 of a row is dH/dlambda.
 // advance: an md step (records row = the device step counter, which the last
 // block to finish advances); otherwise a single point (row 0, counter untouched)
 __global__ void __launch_bounds__(BLOCK) k_reduce(SysPtrs p, int32_t npad, int32_t with_long,
@@ -3558,7 +3555,6 @@ __global__ void __launch_bounds__(BLOCK) k_reduce(SysPtrs p, int32_t npad, int32
     const int32_t step = advance ? *p.step : 0;
     int32_t jb = blockIdx.x;
     const JobDev& J = p.jobs[jb];
-    const int32_t stride = p.nrow_blocks;
     double v[W] = {0};
     // solute atoms' general pairs: per-atom records (short every step, long cached)
     for (int32_t w = J.sol_off + threadIdx.x; w < J.sol_off + J.n_solute_atoms; w += blockDim.x) {
@@ -3590,7 +3586,7 @@ __global__ void __launch_bounds__(BLOCK) k_reduce(SysPtrs p, int32_t npad, int32
         int32_t b1 = (J.atom_off + (advance ? J.n_solute_atoms : J.n_atoms) + per - 1) / per;
 #pragma unroll 2
         for (int32_t b = b0 + threadIdx.x; b < b1; b += blockDim.x) {
-            const double* r = p.rows + ((int64_t)SLOT_EXCL * stride + b) * ROW;
+            const double* r = p.rows + (int64_t)b * ROW;
 #pragma unroll
             for (int c = 0; c < 11; ++c) v[c] += r[c];
             v[12] += r[11];
@@ -3848,7 +3844,7 @@ void launch_vv(const SysPtrs& p, int32_t ncg, int32_t aps, int32_t form, int32_t
         }
     });
 }
-void launch_gen(const SysPtrs& p, int32_t npad, bool lng, int32_t virial, int32_t mixed, int32_t ngsol,
+void launch_gen(const SysPtrs& p, bool lng, int32_t virial, int32_t mixed, int32_t ngsol,
                 hipStream_t s, int32_t part) {
     const bool solv = part != GEN_SOLUTE, solu = part != GEN_SOLVENT;
     // solvent groups, then the solute atoms: a block each of the small solutes, a

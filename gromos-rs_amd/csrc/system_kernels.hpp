@@ -85,7 +85,6 @@ struct SysPtrs {
     float4* xf;                // mixed: the solvent's far_copy (box fractions, offsets, dipole)
     long long* fi_s;           // mixed: int64 fixed-point forces (sorted)
     long long* fi_long_s;      // mixed: twin-range cache
-    int32_t nrow_blocks;       // row stride of the energy partials per slot
     double* f_s;
     double* f_long_s;
     double* f_x;
@@ -170,7 +169,7 @@ void launch_vv_near(const SysPtrs& p, int32_t aps, int32_t form, int32_t virial,
 // ngsol: solvent groups listed in gsol by the last pair search (short passes);
 // part: GEN_ALL, or (mixed short pass) only the solvent or only the solute atoms
 constexpr int32_t GEN_ALL = 0, GEN_SOLVENT = 1, GEN_SOLUTE = 2;
-void launch_gen(const SysPtrs& p, int32_t npad, bool lng, int32_t virial, int32_t mixed, int32_t ngsol,
+void launch_gen(const SysPtrs& p, bool lng, int32_t virial, int32_t mixed, int32_t ngsol,
                 hipStream_t s, int32_t part = GEN_ALL);
 // solv_energy: also the solvent molecules' excluded RF energy (single points;
 // md steps take it in the integrator)
