@@ -96,7 +96,8 @@ void rebox_image(JobImage& im, const Box& box) {
 // of gromos_amd_system), used for admission by footprint
 constexpr int64_t BYTES_PER_ATOM = 2 * 2 * 24 + 7 * 24 + 32 + 16 + 8 + 4 + 8 + 8 + 4 + 12 + 16 + 41 +
                                    ROW * 8 / BLOCK + 1 + 16;
-constexpr int64_t BYTES_PER_CG = 2 * 24 + 16 + 16 + 16 + 4 * 8 + 2 * 8 + 2 * 4 + 8;
+constexpr int64_t BYTES_PER_CG = 2 * 24 + 16 + 16 + 16 + 4 * 8 + 2 * 8 + 2 * 4 + 8 + 16 + 4;   // + s_fix, gen_short
+constexpr int64_t BYTES_PER_CG_TWIN = 11 * 8;   // vv_l
 
 // setup_lincs (constraints.rs:1168-1220): sd[k] = 1 / sqrt(1/m_i + 1/m_j); two
 // constraints a < b sharing an atom (checked first-first, second-first,
@@ -422,7 +423,8 @@ int make_image(const gromos_amd_topology& T, const gromos_amd_params& P, int j, 
     }
     int64_t cells = (int64_t)J.ncell[0] * J.ncell[1] * J.ncell[2];
     im.list_entries = (int64_t)(ncg * partners * 1.25);
-    im.footprint = npad * BYTES_PER_ATOM + (int64_t)T.n_cg * BYTES_PER_CG + 8 * cells +
+    im.footprint = npad * BYTES_PER_ATOM + (int64_t)T.n_cg * (BYTES_PER_CG + (J.twin ? BYTES_PER_CG_TWIN : 0)) +
+                   8 * cells +
                    (int64_t)(ncg * partners * 4.0 * 2.5) + (int64_t)(im.excl.size() + im.o14.size() * 2) * 4 +
                    (int64_t)(2.5 * 1000 * REC * sizeof(double)) + 4096 +
                    (int64_t)im.bonded.atoms.size() * (16 + 32 + 4 + 8 * (12 + BD_EV) + 4 * 4) * 5 / 4;

@@ -63,6 +63,9 @@ def test_job_footprint_host_side():
     # footprint of the 98k-atom water box (per-atom arrays, lists with their
     # growth allowance) stays below 3 KB per atom
     assert rt.Session.footprint(gen.water_32768()) < 3072 * 98304
+    # a twin range's cached records: 88 B a group
+    twin = gen.spc_water_box(1000, seed=1, rcutp=0.8)
+    assert rt.Session.footprint(twin) == fs + 88 * 1000
     bad = gen.spc_water_box(10, seed=1)
     bad.iac = bad.iac.copy()
     bad.iac[0] = bad.n_types       # type out of range
