@@ -107,7 +107,12 @@ constexpr int VV_CHUNK = 16;   // groups per chunk of the solvent pair kernels (
 // environment sets another radius (0: all FP32).
 constexpr double VV_NEAR_R = 0.6;
 constexpr int VV_PARTS = 128;
-constexpr int SOL_WAVE_MIN = 512;   // solute atoms from which a job's take a wave each instead of a block
+// solute atoms from which a job's take a wave each instead of a block of four (k_gen_sol):
+// below, the atoms are too few to fill the chip with a wave each, and their lists are
+// walked faster by four.  Microseconds a launch, block / wave: 512 atoms 14.9 / 23.3
+// in FP64 and 15.2 / 23.7 mixed, 1,536 25.1 / 30.0 and 28.9 / 29.9, 2,048 32.4 / 31.4
+// and 33.4 / 31.4, 4,096 54.6 / 44.5 and 60.3 / 42.8
+constexpr int SOL_WAVE_MIN = 2048;
 constexpr int PRESS_PARTS = 16;   // blocks per pressure-coupled job
 constexpr int PART_W = 13;
 

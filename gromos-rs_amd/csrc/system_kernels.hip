@@ -2358,11 +2358,11 @@ __global__ void __launch_bounds__(BLOCK) k_gen_sv(SysPtrs p, int32_t ngsol) {
 // Energies go to the per-solute-atom record sol_e[(LONG ? nsol : 0) + w] that
 // k_reduce adds per job.  (Eight waves per atom measured slower than four on
 // the 64-job FEP mix: 60 against 46 us per step.)  A job with SOL_WAVE_MIN solute
-// atoms or more fills the chip with a wave per atom, whose sums over the lanes then
-// weigh a quarter (NT = 64; the choice is the job's, so its bits do not depend on
-// the batch): 6,000 atoms in 18,000 waters 70 us in FP64, 280 with a block per atom,
-// IEEE division and square root and the soft-core code in the same kernel.  PERT: the batch has
-// perturbed atoms (the soft-core code's registers only there).
+// atoms or more has enough of them to fill the chip with a wave each, whose sums over
+// the lanes then weigh a quarter (NT = 64; the choice is the job's, so its bits do not
+// depend on the batch): 6,000 atoms in 18,000 waters 70 us in FP64, 280 with a block per
+// atom, IEEE division and square root and the soft-core code in the same kernel.  PERT:
+// the batch has perturbed atoms (the soft-core code's registers only there).
 template <bool LONG, bool MIXED, bool VIR, bool PERT, int NT>
 __global__ void __launch_bounds__(NT) k_gen_sol(SysPtrs p, const int32_t* order, int32_t nsol, int32_t virial) {
     constexpr int NV = ROW + 3;
