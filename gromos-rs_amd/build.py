@@ -3,8 +3,11 @@
     python -m importlib ... or: python gromos-rs_amd/build.py
 
 Flags:
-  -ffp-contract=off            no fused multiply-add: the FP64 path restates the
-                               reference arithmetic operation by operation;
+  -ffp-contract=off            no fused multiply-add but the written ones: the
+                               explicit loops, the excluded, 1-4, soft-core and
+                               covalent terms restate the reference arithmetic
+                               operation by operation, and a job's bits do not
+                               depend on which instantiation of a kernel it meets;
   -Xclang -target-feature -Xclang -packed-fp32-ops
                                keep the compiler from emitting packed FP32 ops.
 """

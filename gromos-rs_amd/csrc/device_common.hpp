@@ -7,8 +7,10 @@
 //   soft-core kernel     crates/gromos-forces/src/nonbonded/perturbed.rs:124-266
 // HIP's double division and sqrt are the correctly rounded IEEE operations and
 // round() rounds half away from zero like f64::round, so each per-pair value of
-// the functions here equals the reference's bit for bit.  (The resident solvent
-// pair kernels take 1/r and the reaction field another way, to the last places.)
+// the functions here equals the reference's bit for bit.  (The resident systems'
+// listed pairs, solvent-solvent and general, take 1/r from the hardware's estimate and
+// a cubic step, and neutral solvent molecules the reaction field through their
+// dipoles: equal to the last places, system_kernels.hip.)
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -49,7 +49,10 @@ __global__ void __launch_bounds__(EXPL_BLOCK) k_fold(const double* part, int64_t
 // pairs holds a few hundred atoms, and a memory atomic per pair side was what the
 // list loops spent their time on: 54 per water pair, 6 per atom pair, colliding on
 // the first atom.  An atom that finds no place within FT_PROBES steps (a list
-// without any locality) goes to memory directly.
+// without any locality) goes to memory directly.  Lists in random order, against the
+// memory atomics alone: 3,000,000 plain pairs of 9,261 waters 850 us (944), 1,781,689
+// molecule pairs 1,385 us (4,343), 9,875 of 216 waters 52 us (69), their 88,875 atom
+// pairs 60 us (60).
 constexpr int FT_PROBES = 16;
 template <int LOG>
 struct ForceTable {

@@ -795,8 +795,8 @@ __device__ __forceinline__ bool has_lj(int i, int j) {
 }
 
 // 1/r in FP64: the hardware estimate (v_rsq_f64, relative error below 2^-22) and one
-// cubic step, y (1 + e/2 + 3 e^2/8) with e = 1 - r2 y^2 (the next term, 5 e^3/16,
-// is below 2^-67), so only the last operations' rounding is left.  Against the
+// cubic step, y (1 + e/2 + 3 e^2/8) with e = 1 - r2 y^2, below 2^-21 (the next term,
+// 5 e^3/16, is below 2^-64), so only the last operations' rounding is left.  Against the
 // IEEE division and square root it replaces (about 30 instructions): 6, of which
 // one quarter rate.
 __device__ __forceinline__ double rsqrt64(double r2) {
@@ -1006,7 +1006,10 @@ __device__ __forceinline__ void vv64_lane(const SysPtrs& p, const JobDev& J, int
     }
 }
 
-// The plain path's solvent pairs (vv64_lane over a molecule's whole list).  VALU
+// The plain path's solvent pairs (vv64_lane over a molecule's whole list).  Forces
+// against the same sums in 80 bits, RMS over boxes of 216 and 2,187 waters: 7.8e-13 and
+// 8.6e-13 kJ/mol/nm, 1.04e-12 and 1.50e-12 with the IEEE operations and the reaction
+// field per atom pair (the Coulomb force's 1/r2 is the plain square of 1/r).  VALU
 // bound: about 295 instructions per listed molecule pair (nine atom pairs), four
 // waves per SIMD.  32,768 waters at 1.4 nm (5.64e7 pair interactions): 119 us, with
 // the IEEE division and square root, the reaction field per atom pair and the
