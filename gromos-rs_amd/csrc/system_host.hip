@@ -1407,7 +1407,7 @@ int md_steps(gromos_amd_system* S, int32_t nsteps, std::vector<double>* rec, std
         HIPCHK(hipMemcpyAsync(S->d_job_step0, S->job_step0.data(), S->job_step0.size() * sizeof(int64_t),
                               hipMemcpyHostToDevice, st));
     // graph replay of the plain steps is opt-in (GROMOS_AMD_GRAPHS=1): on this
-    // runtime it measured 1.5 % slower than separate launches (water_32768)
+    // runtime it is no faster than separate launches (water_32768)
     const char* genv = std::getenv("GROMOS_AMD_GRAPHS");
     S->use_graphs = genv && std::atoi(genv) == 1;
     const char* senv = std::getenv("GROMOS_AMD_SIDE_STREAM");

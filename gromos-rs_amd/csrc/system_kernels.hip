@@ -232,8 +232,8 @@ __device__ __forceinline__ double ref_d2(const Box& b, d3 lo, d3 hi) {
 // a rectangular box a point that is not finite is marked, and distances that may
 // involve one are all taken the reference's way.)
 // Bound by instructions: about 60 vector ones per 64 candidates.  32,768 waters at
-// 1.4 nm: 109 us (156 with FP64 distances and every group's cursors in vector
-// registers); 128 x 4,000 waters at 1.2 nm: 1,041 us (1,544).
+// 1.4 nm: 116 us (156 with FP64 distances and every group's cursors in vector
+// registers); 128 x 4,000 waters at 1.2 nm: 1,047 us (1,544).
 // FILL = false: count only.  FILL = true: write at most cap[k] entries per
 // group, record the true counts and raise *overflow when a group had more.
 // Pair counts: the cell's total goes to the cell's first group, zeros to the
@@ -1107,9 +1107,9 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4
 // FP32 chain over the group's pairs, the virial in FP32 too, 1.738e-4, 2.33e-3, 1.72e-3.
 //
 // VALU bound (about 230 instruction slots per entry, reciprocal square roots
-// counting four; four waves per SIMD).  32,768 waters at 1.4 nm: 77 us (101 with
+// counting four; four waves per SIMD).  32,768 waters at 1.4 nm: 76 us (101 with
 // FP64 shifts, the job's constants in vector registers, int64 sums per group and
-// energies of the canonical side only); 128 x 4,000 waters at 1.2 nm: 721 us
+// energies of the canonical side only); 128 x 4,000 waters at 1.2 nm: 726 us
 // (1,077); 2,187 waters at 1.2 nm with the virial: 21 us (37).
 constexpr int VV_SPREAD = 16;        // a multiple of every lane count
 constexpr double FIX_MAX_L = 40.0;   // nm
