@@ -289,6 +289,7 @@ template <bool FILL, bool RECT>
 __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double near_r2) {
     __shared__ int4 sfix[NBL_PIECE];   // box fractions, original index
     __shared__ int32_t sm[NBL_PIECE], sst[NBL_PIECE], snn[NBL_PIECE];
+    __shared__ double sref[RECT ? 1 : 3][RECT ? 1 : NBL_PIECE];   // other boundaries: reference points
     __shared__ int32_t run_m0[NBL_RUNS], run_off[NBL_RUNS + 1];
     // each wave's own groups (box fractions, original index), read back with a
     // uniform address in the candidate loop: a broadcast through LDS instead of
@@ -301,8 +302,13 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
     if (s0 >= s1) return;     // empty cell: the whole block leaves before any barrier
     const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
     const JobDev& J = p.jobs[p.cg_job[p.s_cg_orig[s0]]];
-    const Box& box = J.box;
-    if ((box.kind == 1) != RECT) return;   // block-uniform, before any barrier
+    if ((J.box.kind == 1) != RECT) return;   // block-uniform, before any barrier
+    // other boundaries reduce every candidate in FP64 with the box: from a copy (the
+    // list's stores would make the compiler read J.box again for each) and points staged
+    // in LDS.  2,744 waters in a truncated octahedron, a rebuild every five steps: 5,180 us
+    // a step, 7,300 with both read from memory
+    const Box box_copy = RECT ? Box{} : J.box;
+    const Box& box = RECT ? J.box : box_copy;
     const double c2s = J.c2s, c2l = J.c2l;
     const int32_t cg_off = J.cg_off, nsol = J.n_solute_cg, aps = J.aps;
     const int32_t nx = J.ncell[0], ny = J.ncell[1], nz = J.ncell[2];
@@ -404,6 +410,11 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
                 if (RECT && mf.w < 0) s_lost = 1;
                 mf.w &= ~FIX_LOST;
                 sfix[q] = mf;
+                if (!RECT) {
+                    sref[0][q] = p.s_ref[3 * m];
+                    sref[RECT ? 0 : 1][q] = p.s_ref[3 * m + 1];
+                    sref[RECT ? 0 : 2][q] = p.s_ref[3 * m + 2];
+                }
                 sm[q] = m;
                 sst[q] = p.s_cg_start[m];
                 snn[q] = p.s_cg_n[m];
@@ -424,6 +435,7 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
                 const int32_t vbase = bcast(vv_base, t), vcap = bcast(vv_end, t) - vbase;
                 int32_t vlo = vbase + bcast(vv_nn, t), vhi = vbase + vcap - 1 - bcast(vv_nf, t);
                 int32_t ns = bcast(gen_ns, t), nl = bcast(gen_nl, t);
+                const d3 ri = RECT ? d3{0.0, 0.0, 0.0} : ld3(p.s_ref, i);
                 for (int32_t cb = 0; cb < plen; cb += WAVE) {
                     const int32_t q = cb + lane;
                     const bool valid = q < plen;
@@ -449,7 +461,7 @@ __global__ void __launch_bounds__(BLOCK) k_nbl(SysPtrs p, int32_t ncell, double 
                             near = !(d2 >= near_r2);
                         }
                     } else {
-                        const d3 r = nim_search(box, ld3(p.s_ref, i), ld3(p.s_ref, sm[qq]));
+                        const d3 r = nim_search(box, ri, d3{sref[0][qq], sref[RECT ? 0 : 1][qq], sref[RECT ? 0 : 2][qq]});
                         const double d2 = r.x * r.x + r.y * r.y + r.z * r.z;
                         in = !(d2 > c2l);
                         lng = d2 > c2s;
