@@ -2161,7 +2161,7 @@ __device__ __forceinline__ void gen_atom32(const SysPtrs& p, int32_t a, int32_t 
     const bool jp = PERT && !LONG && J.has_pert;
     // SOLV (a solvent atom's lane): solvent atoms are never perturbed; of a listed
     // pair with a perturbed first atom the lane takes its own share in FP32, and
-    // of a cached long one its correction in FP64 outside this function (k_gen_sv)
+    // of a cached long one its correction in FP64 elsewhere (k_pert_long)
     const bool po = !SOLV && jp && p.pflag[o];
     PertAtom PA{};
     if (po) PA = pert_atom(p, J, o);
@@ -2321,11 +2321,8 @@ __device__ __forceinline__ void gen_atom32(const SysPtrs& p, int32_t a, int32_t 
 // those pairs' energies and virial belong to the solute atom's block
 // (k_gen_sol): these lanes add none.  (Run beside the solvent pair kernel into
 // a per-group buffer added afterwards, it measured slower: 2.25e11 against
-// 2.33e11 pairs/s on the 64-job FEP mix.)  TWIN: the batch has twin-range jobs with
-// perturbed atoms, whose cached long pairs are corrected every step at the current
-// positions, the solvent atoms' share here (FP64, an instantiation of its own for
-// its registers).
-template <int GSV_LANES, bool PERT, bool TWIN>
+// 2.33e11 pairs/s on the 64-job FEP mix.)
+template <int GSV_LANES, bool PERT>
 __global__ void __launch_bounds__(BLOCK) k_gen_sv(SysPtrs p, int32_t ngsol) {
     constexpr int GSV_SLOT = 4 * GSV_LANES;   // solvent molecules have at most 4 atoms
     const int32_t w = ((int32_t)blockIdx.x * BLOCK + (int32_t)threadIdx.x) / GSV_SLOT;
@@ -2339,21 +2336,6 @@ __global__ void __launch_bounds__(BLOCK) k_gen_sv(SysPtrs p, int32_t ngsol) {
         if (i < p.s_cg_n[k] && !held(p, p.atom_job[p.s2o[sk]])) a = sk + i;
     }
     if (a >= 0) gen_atom32<false, false, true, PERT>(p, a, p.s2o[a], c, GSV_LANES, v, fx, fy, fz);
-    if (TWIN && a >= 0) {
-        const int32_t o = p.s2o[a];
-        const JobDev& J = p.jobs[p.atom_job[o]];
-        int32_t e0 = 0, e1 = 0;
-        if (J.has_pert && J.twin) gen_range(p, p.s_atom_cg[a], true, e0, e1);
-        for (int32_t e = e0 + c; e < e1; e += GSV_LANES) {
-            const uint32_t ent = p.gen_ent[e];
-            if (!(ent & ENT_LONG) || (ent & (ENT_CANON | ENT_VVLONG))) continue;
-            const int32_t m = (int32_t)(ent & ENT_IDX), sm = p.s_cg_start[m], nm = p.s_cg_n[m];
-            for (int32_t b = 0; b < nm; ++b) {
-                const int32_t ob = p.s2o[sm + b];
-                if (p.pflag[ob]) pert_pair_delta(p, J, ob, o, false, v, fx, fy, fz);
-            }
-        }
-    }
 #pragma unroll
     for (int m = 1; m < GSV_LANES; m <<= 1) {
         fx += __shfl_xor(fx, m, WAVE);
@@ -2365,6 +2347,59 @@ __global__ void __launch_bounds__(BLOCK) k_gen_sv(SysPtrs p, int32_t ngsol) {
         p.fi_s[3 * a + 1] += to_fx(fy);
         p.fi_s[3 * a + 2] += to_fx(fz);
     }
+}
+
+// Mixed precision, twin-range jobs with perturbed atoms: the solvent atoms' share of
+// the cached long pairs' correction, taken every step at the current positions (FP64;
+// the solute atoms take theirs and the energies in k_gen_sol).  A wave per listed
+// group scans its long entries; the few perturbed partners among 64 entries are moved
+// to the first lanes, and four lanes each take them, a lane an atom of the molecule:
+// a soft-core pair is a chain of some thousand cycles, so no lane should take two in
+// a row.  Summed by a fixed butterfly and added after k_gen_sv.  A 600-atom chain, every
+// seventh atom perturbed, in 1,500 waters: 163 us a step, 161 without the correction,
+// 356 with sixteen lanes a group, each its own entries with all the molecule's atoms.
+__global__ void __launch_bounds__(BLOCK) k_pert_long(SysPtrs p, int32_t ngsol) {
+    const int32_t w = __builtin_amdgcn_readfirstlane((int32_t)(blockIdx.x * (BLOCK / WAVE) + threadIdx.x / WAVE));
+    if (w >= ngsol) return;
+    const int lane = threadIdx.x & (WAVE - 1), i = lane & 3;
+    const int32_t k = __builtin_amdgcn_readfirstlane(p.gsol[w]);
+    const int32_t sk = p.s_cg_start[k], nk = p.s_cg_n[k], job = p.atom_job[p.s2o[sk]];
+    const JobDev& J = p.jobs[job];
+    if (!J.has_pert || !J.twin || held(p, job)) return;   // the whole wave
+    int32_t e0, e1;
+    gen_range(p, k, true, e0, e1);
+    const int32_t own = i < nk ? p.s2o[sk + i] : -1;
+    double f[3] = {0.0, 0.0, 0.0}, v[ROW] = {0};
+    for (int32_t eb = e0; eb < e1; eb += WAVE) {
+        int32_t sm = 0, nm = 0;
+        if (eb + lane < e1) {
+            const uint32_t ent = p.gen_ent[eb + lane];
+            const int32_t m = (int32_t)(ent & ENT_IDX);
+            if ((ent & ENT_LONG) && !(ent & (ENT_CANON | ENT_VVLONG)) && p.cg_pert[p.s_cg_orig[m]]) {
+                sm = p.s_cg_start[m];
+                nm = p.s_cg_n[m];
+            }
+        }
+        for (int32_t b = 0; __any(b < nm); ++b) {
+            const int32_t ob = b < nm ? p.s2o[sm + b] : -1;
+            const bool on = ob >= 0 && p.pflag[ob];
+            const uint64_t mask = __ballot(on);
+            const int32_t n = (int32_t)__popcll(mask);
+            const int32_t packed =
+                __builtin_amdgcn_ds_permute(4 * (on ? lane_rank(mask) : n + lane_rank(~mask)), ob);
+            for (int32_t q = 0; q < n; q += WAVE / 4) {
+                const int32_t partner = __shfl(packed, min(q + lane / 4, WAVE - 1), WAVE);
+                if (q + lane / 4 < n && own >= 0) pert_pair_delta(p, J, partner, own, false, v, f[0], f[1], f[2]);
+            }
+        }
+    }
+#pragma unroll
+    for (int m = 4; m < WAVE; m <<= 1)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) f[d] += __shfl_xor(f[d], m, WAVE);
+    if (lane < nk)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) p.fi_s[3 * (sk + lane) + d] += to_fx(f[d]);
 }
 
 // Solute atoms: one block of NT lanes per atom (global solute index w = order[block],
@@ -3894,9 +3929,11 @@ void launch_gen(const SysPtrs& p, bool lng, int32_t virial, int32_t mixed, int32
         constexpr int32_t GPB = BLOCK / (4 * 2);   // groups per block
         const dim3 g((unsigned)((ngsol + GPB - 1) / GPB));
         if (solv && ngsol > 0) {
-            if (p.pert_twin) hipLaunchKernelGGL((k_gen_sv<2, true, true>), g, dim3(BLOCK), 0, s, p, ngsol);
-            else if (pert) hipLaunchKernelGGL((k_gen_sv<2, true, false>), g, dim3(BLOCK), 0, s, p, ngsol);
-            else hipLaunchKernelGGL((k_gen_sv<2, false, false>), g, dim3(BLOCK), 0, s, p, ngsol);
+            if (pert) hipLaunchKernelGGL((k_gen_sv<2, true>), g, dim3(BLOCK), 0, s, p, ngsol);
+            else hipLaunchKernelGGL((k_gen_sv<2, false>), g, dim3(BLOCK), 0, s, p, ngsol);
+            constexpr int32_t PLB = BLOCK / WAVE;   // groups per block
+            if (p.pert_twin)
+                hipLaunchKernelGGL(k_pert_long, dim3((unsigned)((ngsol + PLB - 1) / PLB)), dim3(BLOCK), 0, s, p, ngsol);
         }
         if (solu) {
             if (virial && pert) GAMD_SOL(false, true, true, true, 1);
