@@ -4,7 +4,7 @@
 //                 k_nbl<FILL> / k_totals / k_job_pairs
 //                                    StandardPairlistAlgorithm semantics
 //                                    (pairlist.rs:183-442) on a cell grid
-//  forces         k_gather, k_vv / k_vv_mx / k_vv_nr, k_gen_sv64 / k_gen_sv / k_gen_sol, k_long,
+//  forces         k_gather, k_vv / k_vv_mx / k_vv_nr, k_gen_sv64 / k_gen_sv / k_pert_long / k_gen_sol, k_long,
 //                 k_excl14, k_assemble
 //                                    (innerloops.rs:105-309, excluded.rs:25-206,
 //                                     forcefield.rs:420-756)
